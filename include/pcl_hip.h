@@ -89,10 +89,11 @@ int pcl_stream_destroy(void *stream);
  * activations, the INT8 GEMM's tile counters (64 bytes: the persistent kernel
  * of outputs past 256 MiB hands its tiles out from them, so calls on one
  * stream must not overlap -- stream order guarantees it), pcl_head_ce's
- * logits chunk, and the realigned copies of
- * misaligned FP32 operands that pcl_sgemm makes for products of >= 2^30
- * multiply-adds (for the trainer's head backward over 4096 x 50257 logits
- * about 0.8 GB). pcl_release_scratch waits for the stream (hip_stream, NULL =
+ * logits chunk, and the split
+ * operands of large FP32 products on the f16 matrix cores (pcl_sgemm; 4 bytes
+ * per element of both: for the trainer's head backward over 4096 x 50257
+ * logits about 0.8 GB; where they cannot be allocated such a product runs on
+ * the f32 matrix cores instead). pcl_release_scratch waits for the stream (hip_stream, NULL =
  * null stream) and frees these buffers; the next call allocates again. It
  * fails with PCL_ERR_INVALID_ARG on a stream a graph was captured on (the
  * graph may use them; pcl_stream_destroy frees them). Calls on the stream
@@ -228,8 +229,13 @@ void ce_fwd_bwd(const float *logits, const int *targets, float *dlogits, float *
 #define PCL_OP_N 0 /* operand stored as written: A is M x K, B is K x N */
 #define PCL_OP_T 1 /* operand stored transposed: A is K x M, B is N x K */
 
-/* FP32 GEMM on the f32 MFMA: C(M,N) = (accumulate ? C : 0) + op(A)·op(B) + bias.
- * Decode shapes (M <= 8, opA == N) run the HBM-bound GEMV kernels instead.
+/* FP32 GEMM: C(M,N) = (accumulate ? C : 0) + op(A)·op(B) + bias, on the f32 MFMA;
+ * large products (from about 2^30 multiply-adds on) on the f16 MFMA, each
+ * operand as a sum of two f16 values under a power-of-two scale per row of op(A)
+ * and column of op(B), all sums in fp32: as exact as the f32 form or more so
+ * for rows whose elements span up to 2^17; an element below 2^-39 of its row's
+ * largest counts as 0. Rows and columns with infinities or NaN give the IEEE
+ * result. Decode shapes (M <= 8, opA == N) run the HBM-bound GEMV kernels.
  * Replaces tensor.c:34-53, train.c:181-252/412-447, gpu_kernels.cu:112-138. */
 int pcl_sgemm(int opA, int opB, int M, int N, int K, const float *A, int lda, const float *B,
               int ldb, const float *bias, int accumulate, float *C, int ldc, void *stream);

@@ -14,6 +14,7 @@ namespace pcl {
 struct Workspace {
     void *buf = nullptr;  // bytes_cap bytes
     size_t bytes_cap = 0;
+    void *operands = nullptr;  // the split operands of a GEMM on the f16 matrix cores
 };
 
 // Split-K GEMV geometry chosen by the launchers; the shim sizes the workspace.
@@ -26,6 +27,13 @@ struct GemvPlan {
 };
 
 // ---- FP32 GEMM (sgemm.hip) ----
+// The same product on the f16 matrix cores (sgemm_split.hip): tile and K split,
+// bytes of the split operands (0: the shape has no such form) and of the
+// partial products.
+struct SgemmF16Plan {
+    int cfg = 0, splits = 1, kchunk = 0;
+    size_t op_bytes = 0, part_bytes = 0;
+};
 // Tile configuration and K split chosen for a shape; with splits > 1 the
 // partial products ([splits][M][N] fp32, part_bytes) go to the workspace and a
 // second kernel adds them in split order.
@@ -34,7 +42,10 @@ struct SgemmPlan {
     int splits;
     int kchunk;         // K per split (a multiple of 64 when split)
     size_t part_bytes;  // workspace bytes (0 when splits == 1)
+    SgemmF16Plan f16 = {};
+    bool use_f16 = false;  // launch_sgemm runs f16 (workspace: f16.part_bytes and operands)
 };
+SgemmF16Plan plan_sgemm_f16(int M, int N, int K);
 // a_kcontig: op(A) is K-contiguous (row-major A, no transpose), which the
 // 32x64 small-grid configuration needs
 SgemmPlan plan_sgemm(int M, int N, int K, bool a_kcontig = false);
@@ -51,6 +62,12 @@ hipError_t launch_sgemm(const SgemmPlan &p, bool a_kcontig, bool b_kcontig, int 
                         int accumulate, float *C, long ldc, const Workspace &ws,
                         hipStream_t stream, int epi = EPI_NONE, const float *aux_in = nullptr,
                         float *aux_out = nullptr, long ld_aux = 0);
+// The second pass of a K split: C = (accumulate ? C : 0) + sum of the partial
+// products P[splits][M][N] in split order + bias, then the epilogue.
+hipError_t launch_splitk_reduce(const float *P, int splits, int M, int N, const float *bias, float *C, long ldc,
+                                int accumulate, int epi, const float *aux_in, float *aux_out, long ld_aux,
+                                hipStream_t stream);
+
 // dst (rows x cols, ldd % 4 == 0, 16-byte aligned) <- src (lds, any alignment)
 hipError_t launch_copy_rows(float *dst, long ldd, const float *src, long lds, int rows, int cols,
                             hipStream_t stream);

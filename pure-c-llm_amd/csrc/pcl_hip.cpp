@@ -132,9 +132,10 @@ struct StreamScratch {
     pcl::Workspace ws;
     void *aux = nullptr;  // padded INT8 activations; head_ce's logits chunk and row losses
     size_t aux_cap = 0;
-    // Realigned copies of misaligned FP32 GEMM operands (sgemm_realigned).
-    // Kept apart from aux: pcl_head_ce holds its logits chunk in aux while it
-    // calls pcl_sgemm, which may realign on the same stream.
+    // Split operands of FP32 GEMMs on the f16 matrix cores (sgemm_f16), or
+    // realigned copies of misaligned ones (sgemm_realigned). Kept apart from
+    // aux: pcl_head_ce holds its logits chunk in aux while it calls pcl_sgemm,
+    // which may need them on the same stream.
     void *realign = nullptr;
     size_t realign_cap = 0;
     unsigned *amax = nullptr;  // per-tensor amax bits
@@ -782,7 +783,60 @@ int pcl_sgemv_noalloc(int opW, int M, int N, int K, const float *X, int ldx, con
     return PCL_OK;
 }
 
-// A large product whose operands miss the LDS-DMA kernel's requirements
+// Operands the LDS-DMA kernels of sgemm.hip read as they are.
+static bool dma_operands(int opA, int opB, int M, int N, int K, const float *A, int lda, const float *B, int ldb) {
+    const bool a_kc = opA == PCL_OP_N, b_kc = opB == PCL_OP_T;  // K-contiguous operands
+    return aligned16(A) && aligned16(B) && lda % 4 == 0 && ldb % 4 == 0 && (a_kc ? K % 4 == 0 : M % 4 == 0) &&
+           (b_kc ? K % 4 == 0 : N % 4 == 0) && K % 32 == 0;
+}
+
+// Products that the f16 matrix cores take (plan.f16, sgemm_split.hip): their
+// split pass over the operands costs 10-25 us, so they have to be large. From
+// 1.25 * 2^30 multiply-adds on over operands the f32 kernels read by DMA (928 x
+// 544 x 3840 61.5 -> 45.6 us, 544 x 3136 x 864 36.9 -> 30.3, but 1024^3 22.4 ->
+// 27), from 2^29 on over others (627 x 1191 x 1058 41.6 -> 27.6 us, 591 x 1560
+// x 586 26.2 -> 25.3; 529 x 2819 x 141 and the like gain, 112 x 2172 x 1534 is
+// level).
+static bool f16_pays(const pcl::SgemmPlan &p, int opA, int opB, int M, int N, int K, const float *A, int lda,
+                     const float *B, int ldb) {
+    const double macs = (double)M * N * K;
+    return p.f16.op_bytes > 0 &&
+           macs >= (dma_operands(opA, opB, M, N, K, A, lda, B, ldb) ? 1.25 * (1L << 30) : 1.0 * (1L << 29));
+}
+
+// The product on the f16 matrix cores. Returns 1, with nothing enqueued, where
+// the caller has to take the f32 ones instead: scratch that cannot be had (the
+// f32 kernels need little or none), and scratch that would have to grow while
+// the stream is captured other than by pcl_graph_begin, where an allocation
+// can end the capture.
+static int sgemm_f16(pcl::SgemmPlan p, int opA, int opB, int M, int N, int K, const float *A, int lda, const float *B,
+                     int ldb, const float *bias, int accumulate, float *C, int ldc, hipStream_t s,
+                     int epi = PCL_EPI_NONE, const float *aux_in = nullptr, float *aux_out = nullptr, int ld_aux = 0) {
+    ScratchLease sc;
+    PCL_OK_OR_RETURN(get_scratch(s, 0, 0, &sc));
+    if (p.f16.part_bytes > sc->ws.bytes_cap || p.f16.op_bytes > sc->realign_cap) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (!t_capturing && (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)) {
+            (void)hipGetLastError();
+            return 1;
+        }
+        const int st = get_scratch(s, p.f16.part_bytes, 0, &sc, p.f16.op_bytes);
+        if (st == PCL_ERR_OOM) {
+            (void)hipGetLastError();
+            pcl_clear_error();
+            return 1;
+        }
+        if (st != PCL_OK) return st;
+    }
+    p.use_f16 = true;
+    pcl::Workspace ws = sc->ws;
+    ws.operands = sc->realign;
+    HIP_OK(pcl::launch_sgemm(p, opA == PCL_OP_N, opB == PCL_OP_T, M, N, K, A, lda, B, ldb, bias, accumulate, C, ldc, ws,
+                             s, epi, aux_in, aux_out, ld_aux));
+    return PCL_OK;
+}
+
+// A large product left on the f32 matrix cores whose operands miss the LDS-DMA kernel's requirements
 // (16-byte aligned rows, contiguous extents a multiple of 4 floats, K a
 // multiple of 32), e.g. the trainer's head backward over 50257-float logits
 // rows (train_kaggle.cu:173-174 through gemm_nn / gemm_tn): each misaligned
@@ -859,17 +913,15 @@ int pcl_sgemm(int opA, int opB, int M, int N, int K, const float *A, int lda, co
     if (M <= 8 && opA == PCL_OP_N)
         return pcl_sgemv(opB, M, N, K, A, lda, B, ldb, bias, accumulate, C, ldc, stream);
     hipStream_t s = pick(stream);
-    if (K > 0 && (double)M * N * K >= (double)(1L << 30)) {
-        const bool a_kc = opA == PCL_OP_N, b_kc = opB == PCL_OP_T;
-        const bool dma_ok = aligned16(A) && aligned16(B) && lda % 4 == 0 && ldb % 4 == 0 &&
-                            (a_kc ? K % 4 == 0 : M % 4 == 0) && (b_kc ? K % 4 == 0 : N % 4 == 0) &&
-                            K % 32 == 0;
-        if (!dma_ok) {
-            const int st = sgemm_realigned(opA, opB, M, N, K, A, lda, B, ldb, bias, accumulate, C, ldc, s);
-            if (st != 1) return st;
-        }
-    }
     pcl::SgemmPlan p = pcl::plan_sgemm(M, N, K, opA == PCL_OP_N);
+    if (f16_pays(p, opA, opB, M, N, K, A, lda, B, ldb)) {
+        const int st = sgemm_f16(p, opA, opB, M, N, K, A, lda, B, ldb, bias, accumulate, C, ldc, s);
+        if (st != 1) return st;
+    }
+    if (K > 0 && (double)M * N * K >= (double)(1L << 30) && !dma_operands(opA, opB, M, N, K, A, lda, B, ldb)) {
+        const int st = sgemm_realigned(opA, opB, M, N, K, A, lda, B, ldb, bias, accumulate, C, ldc, s);
+        if (st != 1) return st;
+    }
     ScratchLease sc;
     PCL_OK_OR_RETURN(get_scratch(s, p.part_bytes, 0, &sc));
     HIP_OK(pcl::launch_sgemm(p, opA == PCL_OP_N, opB == PCL_OP_T, M, N, K, A, lda, B, ldb, bias,
@@ -914,6 +966,11 @@ int pcl_sgemm_ex(int opA, int opB, int M, int N, int K, const float *A, int lda,
     PCL_OK_OR_RETURN(do_init());
     hipStream_t s = pick(stream);
     pcl::SgemmPlan p = pcl::plan_sgemm(M, N, K, opA == PCL_OP_N);
+    if (f16_pays(p, opA, opB, M, N, K, A, lda, B, ldb)) {
+        const int st = sgemm_f16(p, opA, opB, M, N, K, A, lda, B, ldb, bias, 0, C, ldc, s, epilogue, aux_in,
+                                 epilogue == PCL_EPI_GELU ? aux_out : nullptr, ld_aux);
+        if (st != 1) return st;
+    }
     ScratchLease sc;
     PCL_OK_OR_RETURN(get_scratch(s, p.part_bytes, 0, &sc));
     HIP_OK(pcl::launch_sgemm(p, opA == PCL_OP_N, opB == PCL_OP_T, M, N, K, A, lda, B, ldb, bias, 0,
@@ -1575,21 +1632,24 @@ int pcl_head_ce(const float *lnf, const float *wte, const int *targets, int M, i
     PCL_OK_OR_RETURN(get_scratch(s, 0, loss_off + sizeof(double) * (size_t)M, &sc));
     float *lg = static_cast<float *>(sc->aux);
     double *rl = reinterpret_cast<double *>(static_cast<char *>(sc->aux) + loss_off);
-    const int Vm = V / 64 * 64, Vr = V - Vm, L = (int)ldp;
+    const int L = (int)ldp;
     for (int m0 = 0; m0 < M; m0 += (int)mc) {
         const int mm = (int)(M - m0 < mc ? M - m0 : mc);
         const float *x = lnf + (size_t)m0 * D;
         // train.c:412-423 on the chunk, then :449-465 in place
         PCL_OK_OR_RETURN(pcl_sgemm(PCL_OP_N, PCL_OP_T, mm, V, D, x, D, wte, D, nullptr, 0, lg, L, s));
         HIP_OK(pcl::launch_cross_entropy(lg, ldp, targets + m0, lg, ldp, mm, V, L, M, rl + m0, s));
-        if (d_lnf) {  // train.c:426-435 (set): K = V in two parts
+        // the vocabulary in two parts on the f32 matrix cores, whole on the f16 ones
+        const bool f16 = f16_pays(pcl::plan_sgemm(mm, D, V), PCL_OP_N, PCL_OP_N, mm, D, V, lg, L, wte, D);
+        const int Vm = f16 ? V : V / 64 * 64, Vr = V - Vm;
+        if (d_lnf) {  // train.c:426-435 (set): K = V
             float *dx = d_lnf + (size_t)m0 * D;
             PCL_OK_OR_RETURN(pcl_sgemm(PCL_OP_N, PCL_OP_N, mm, D, Vm, lg, L, wte, D, nullptr, 0, dx, D, s));
             if (Vr)
                 PCL_OK_OR_RETURN(pcl_sgemm(PCL_OP_N, PCL_OP_N, mm, D, Vr, lg + Vm, L, wte + (size_t)Vm * D,
                                            D, nullptr, 1, dx, D, s));
         }
-        if (dwte) {  // train.c:436-446 (accumulate): vocabulary rows in two parts
+        if (dwte) {  // train.c:436-446 (accumulate): vocabulary rows
             if (Vm)
                 PCL_OK_OR_RETURN(pcl_sgemm(PCL_OP_T, PCL_OP_N, Vm, D, mm, lg, L, x, D, nullptr, 1, dwte, D, s));
             if (Vr)

@@ -22,11 +22,9 @@
 // per chunk. The sum over k is unchanged; only fp32 rounding order differs
 // from the reference's sequential loop (checked to 1e-4 in the tests).
 #include "internal.h"
+#include "sgemm_common.h"
 
 namespace pcl {
-
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int SG_PAD_K = 4;   // floats of padding per K-contiguous LDS row
 constexpr int SG_PAD_MN = 4;  // floats of padding per MN-contiguous LDS row
@@ -293,33 +291,6 @@ __global__ __launch_bounds__(256 * KG) void sgemm_mfma_kernel(
     }
 }
 
-// ---------------------------------------------------------------------------
-// Epilogues (train.c:314-333 and gpu_kernels.cu:228-243 tanh-GELU, the
-// residual adds of train.c:522/527): applied to v = acc + bias.
-constexpr float GELU_C = 0.7978845608028654f;  // sqrt(2/pi)
-__device__ __forceinline__ float gelu_f(float x) {
-    return 0.5f * x * (1.0f + tanhf(GELU_C * (x + 0.044715f * x * x * x)));
-}
-__device__ __forceinline__ float gelu_grad(float x) {
-    const float t = tanhf(GELU_C * (x + 0.044715f * x * x * x));
-    const float dudx = GELU_C * (1.0f + 3.0f * 0.044715f * x * x);
-    return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * dudx;
-}
-// EPI_GELU: aux_out (if set) <- v, C <- gelu(v); EPI_RESID: C <- aux_in + v;
-// EPI_GELU_BWD: C <- v * gelu'(aux_in)
-template <int EPI>
-__device__ __forceinline__ float apply_epi(float v, const float *aux_in, float *aux_out, long ai) {
-    if constexpr (EPI == EPI_GELU) {
-        if (aux_out) aux_out[ai] = v;
-        return gelu_f(v);
-    } else if constexpr (EPI == EPI_RESID) {
-        return aux_in[ai] + v;
-    } else if constexpr (EPI == EPI_GELU_BWD) {
-        return v * gelu_grad(aux_in[ai]);
-    }
-    return v;
-}
-
 // The same epilogue as a separate pass over an M x N product already in C
 // (operands the fused kernels do not take: unaligned, split K, other layouts).
 // Grid (ceil(N / 256), M).
@@ -415,20 +386,6 @@ hipError_t launch_copy_rows(float *dst, long ldd, const float *src, long lds, in
 // next tile's fragments, then this tile's MFMAs. Requires K % 32 == 0 and the
 // 16-byte vector conditions of the register-staged kernel.
 constexpr int SD_BK = 32;
-
-template <int OFF>
-__device__ __forceinline__ void sd_read128(v4f &r, unsigned addr) {
-    static_assert(OFF >= 0 && OFF < 65536, "ds_read offset field");
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "i"(OFF));
-}
-template <int OFF>
-__device__ __forceinline__ void sd_read32(float &r, unsigned addr) {
-    static_assert(OFF >= 0 && OFF < 65536, "ds_read offset field");
-    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "i"(OFF));
-}
-__device__ __forceinline__ void sd_fence(v4f &r) { asm volatile("" : "+v"(r)); }
-__device__ __forceinline__ void sd_fence(float &r) { asm volatile("" : "+v"(r)); }
-constexpr int sd_waitcnt_vm(int n) { return (n & 15) | (((n >> 4) & 3) << 14) | (7 << 4) | (15 << 8); }
 
 // One operand's part of a ring stage: SUB consecutive K tiles of ROWS (M or
 // N) x SD_BK (K) floats, tile s at byte SUBB * s of the stage.
@@ -1151,6 +1108,14 @@ __global__ void sgemm_splitk_reduce_kernel(const float *__restrict__ P, int spli
     *c = out;
 }
 
+hipError_t launch_splitk_reduce(const float *P, int splits, int M, int N, const float *bias, float *C, long ldc,
+                                int accumulate, int epi, const float *aux_in, float *aux_out, long ld_aux,
+                                hipStream_t stream) {
+    hipLaunchKernelGGL(sgemm_splitk_reduce_kernel, dim3((unsigned)((N + 255) / 256), (unsigned)M), dim3(256), 0,
+                       stream, P, splits, M, N, bias, C, ldc, accumulate, epi, aux_in, aux_out, ld_aux);
+    return hipGetLastError();
+}
+
 template <int BM, int BN, int BK, int KG, int PF, bool A_KC, bool B_KC>
 static hipError_t launch_cfg(bool vec, int M, int N, int K, int splits, int kchunk,
                              const float *A, long lda, const float *B, long ldb, const float *bias,
@@ -1180,6 +1145,7 @@ enum SgemmCfg {
 
 SgemmPlan plan_sgemm(int M, int N, int K, bool a_kcontig) {
     SgemmPlan p{SG_64_KG2, 1, K > 0 ? K : 1, 0};
+    p.f16 = plan_sgemm_f16(M, N, K);
     const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
     const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
     // Grids too small for 256 CUs with a short K (the grown model's prefill
@@ -1431,10 +1397,8 @@ static hipError_t dispatch_layout(const SgemmPlan &p, int M, int N, int K, const
         break;
     }
     if (e != hipSuccess || !split) return e;
-    hipLaunchKernelGGL(sgemm_splitk_reduce_kernel, dim3((unsigned)((N + 255) / 256), (unsigned)M),
-                       dim3(256), 0, stream, static_cast<const float *>(ws.buf), p.splits, M, N, bias,
-                       C, ldc, accumulate, epi, aux_in, aux_out, ld_aux);
-    return hipGetLastError();
+    return launch_splitk_reduce(static_cast<const float *>(ws.buf), p.splits, M, N, bias, C, ldc, accumulate,
+                                epi, aux_in, aux_out, ld_aux, stream);
 }
 
 hipError_t launch_sgemm(const SgemmPlan &p, bool a_kcontig, bool b_kcontig, int M, int N, int K,
@@ -1442,6 +1406,9 @@ hipError_t launch_sgemm(const SgemmPlan &p, bool a_kcontig, bool b_kcontig, int 
                         int accumulate, float *C, long ldc, const Workspace &ws,
                         hipStream_t stream, int epi, const float *aux_in, float *aux_out,
                         long ld_aux) {
+    if (p.use_f16)
+        return launch_sgemm_f16(p.f16, a_kcontig, b_kcontig, M, N, K, A, lda, B, ldb, bias, accumulate, C, ldc, ws,
+                                stream, epi, aux_in, aux_out, ld_aux);
     if (a_kcontig && !b_kcontig)
         return dispatch_layout<true, false>(p, M, N, K, A, lda, B, ldb, bias, accumulate, C, ldc, ws,
                                             stream, epi, aux_in, aux_out, ld_aux);
