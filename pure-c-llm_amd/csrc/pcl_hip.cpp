@@ -1093,7 +1093,9 @@ int attn_bwd_common(const char *fn, float *dQ, float *dK, float *dV, int ld_grad
         dS = static_cast<float *>(sc->ws.buf);
     }
     HIP_OK(pcl::launch_attn_bwd(dAtt, ld_att, Q, K, V, ld, probs, dS, dQ, dK, dV, ld_grad, B, T, H,
-                                dh, 1.0f / sqrtf((float)dh), accumulate, s, att, ld_o));
+                                dh, 1.0f / sqrtf((float)dh),
+                                (accumulate ? pcl::ATTN_ACCUMULATE : 0) | (scratch ? pcl::ATTN_KEEP_DS : 0), s, att,
+                                ld_o));
     return PCL_OK;
 }
 }  // namespace
