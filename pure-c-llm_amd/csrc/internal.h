@@ -62,11 +62,6 @@ hipError_t launch_sgemm(const SgemmPlan &p, bool a_kcontig, bool b_kcontig, int 
                         int accumulate, float *C, long ldc, const Workspace &ws,
                         hipStream_t stream, int epi = EPI_NONE, const float *aux_in = nullptr,
                         float *aux_out = nullptr, long ld_aux = 0);
-// The second pass of a K split: C = (accumulate ? C : 0) + sum of the partial
-// products P[splits][M][N] in split order + bias, then the epilogue.
-hipError_t launch_splitk_reduce(const float *P, int splits, int M, int N, const float *bias, float *C, long ldc,
-                                int accumulate, int epi, const float *aux_in, float *aux_out, long ld_aux,
-                                hipStream_t stream);
 
 // dst (rows x cols, ldd % 4 == 0, 16-byte aligned) <- src (lds, any alignment)
 hipError_t launch_copy_rows(float *dst, long ldd, const float *src, long lds, int rows, int cols,
