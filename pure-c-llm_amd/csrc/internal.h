@@ -29,9 +29,14 @@ struct GemvPlan {
 // ---- FP32 GEMM (sgemm.hip) ----
 // The same product on the f16 matrix cores (sgemm_split.hip): tile and K split,
 // bytes of the split operands (0: the shape has no such form) and of the
-// partial products.
-struct SgemmF16Plan {
+// partial products. With cut_m or cut_n, rows or columns from there on are a
+// launch of their own, with the tile and K split of `rest`.
+struct SgemmF16Part {
     int cfg = 0, splits = 1, kchunk = 0;
+};
+struct SgemmF16Plan {
+    SgemmF16Part main, rest;
+    int cut_m = 0, cut_n = 0;
     size_t op_bytes = 0, part_bytes = 0;
 };
 // Tile configuration and K split chosen for a shape; with splits > 1 the

@@ -527,26 +527,71 @@ struct SplitTile {
 static const SplitTile SPLIT_TILES[] = {{256, 256, 256, 10.f, 2.2f},  {256, 192, 256, 8.f, 1.85f},
                                         {256, 128, 256, 6.f, 1.13f},  {128, 128, 512, 5.f, 1.28f},
                                         {128, 128, 256, 5.f, 0.73f},  {64, 128, 256, 4.f, 0.42f}};
+constexpr double SPLIT_CUT_US = 4, SPLIT_CUT_GAIN = 0.9;  // a second launch, and the share of the time it has to save
+
+constexpr int SPLIT_STEP = SPLIT_BK * SPLIT_KUNITS;  // a K split's granularity
+static double split_us(const SplitTile &t, long tiles, int chunk) {
+    return (double)((tiles + t.per_round - 1) / t.per_round) * (t.edge + t.unit * SPLIT_KUNITS * chunk);
+}
+
+// The best tile and K split of one launch, and its time in us.
+static double plan_part(int M, int N, int K, SgemmF16Part &p) {
+    const int steps = (K + SPLIT_STEP - 1) / SPLIT_STEP;
+    double best = 1e30;
+    for (int c = 0; c < SPLIT_CFGS; c++)
+        for (int z = 1; z <= 16 && z * 4 <= steps + 3; z++) {
+            const SplitTile &t = SPLIT_TILES[c];
+            const int chunk = (steps + z - 1) / z;
+            double us = split_us(t, (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * z, chunk);
+            if (z > 1) us += 4 + (2 * z + 1) * 1e-6 * M * N;
+            if (us < best) best = us, p.cfg = c, p.splits = z, p.kchunk = chunk * SPLIT_STEP;
+        }
+    p.splits = (K + p.kchunk - 1) / p.kchunk;
+    return best;
+}
 
 SgemmF16Plan plan_sgemm_f16(int M, int N, int K) {
     SgemmF16Plan p;
     // Short sums: below 96 terms the two forms' errors meet (measured 1.1e-7 of
     // the result at K = 69, both). Narrow outputs leave most of a tile idle.
     if (K < 96 || M < 128 || N < 128) return p;
-    constexpr int STEP = SPLIT_BK * SPLIT_KUNITS;
-    const int steps = (K + STEP - 1) / STEP;
-    double best = 1e30;
-    for (int c = 0; c < SPLIT_CFGS; c++)
-        for (int z = 1; z <= 16 && z * 4 <= steps + 3; z++) {
+    const double whole = plan_part(M, N, K, p.main);
+    // Several rounds of tiles of which the last is mostly idle: the rows or
+    // columns past the whole rounds (at most an eighth) become a launch of their
+    // own, over smaller tiles and K splits that fill the chip, where that is
+    // expected to save a tenth of the time, with tiles no smaller than before.
+    // 50257 x 1024 x 4096 1373 -> 1208 us (6.2 rounds of 256x128 -> 3 of 256x256),
+    // 2253 x 7717 x 799 127 -> 107, 4096 x 4097 x 700 105 -> 85, 4143 x 4187 x 155
+    // 51 -> 48, eight other shapes 4-17% less. Not for a single round that does
+    // not fill the chip: its tiles run at a higher clock (3521 x 2622 x 1995 125 us
+    // whole and 132 cut, 3006 x 2706 x 1877 114 both ways). Nor from 256x256 to
+    // smaller tiles, which read more (4883 x 5197 x 2006 307 us whole and 314 cut).
+    const SplitTile &t0 = SPLIT_TILES[p.main.cfg];
+    const long tiles0 = (long)((M + t0.bm - 1) / t0.bm) * ((N + t0.bn - 1) / t0.bn);
+    double best = whole * SPLIT_CUT_GAIN;
+    const int steps = (K + SPLIT_STEP - 1) / SPLIT_STEP;
+    int cut_cfg = -1;
+    for (int c = 0; c <= p.main.cfg && p.main.splits == 1 && tiles0 > t0.per_round; c++)
+        for (int cols = 0; cols < 2; cols++) {
             const SplitTile &t = SPLIT_TILES[c];
-            const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * z;
-            const int chunk = (steps + z - 1) / z;
-            double us = (double)((tiles + t.per_round - 1) / t.per_round) * (t.edge + t.unit * SPLIT_KUNITS * chunk);
-            if (z > 1) us += 4 + (2 * z + 1) * 1e-6 * M * N;
-            if (us < best) best = us, p.cfg = c, p.splits = z, p.kchunk = chunk * STEP;
+            const long nm = (M + t.bm - 1) / t.bm, nn = (N + t.bn - 1) / t.bn, rounds = nm * nn / t.per_round;
+            const long keep = rounds * t.per_round / (cols ? nm : nn);  // whole rows or columns of tiles
+            const long cut = keep * (cols ? t.bn : t.bm), len = cols ? N : M;
+            if (cut >= len || cut < len - len / 8) continue;
+            SgemmF16Part rest;
+            const double us = split_us(t, keep * (cols ? nm : nn), steps) + SPLIT_CUT_US +
+                              (cols ? plan_part(M, N - (int)cut, K, rest) : plan_part(M - (int)cut, N, K, rest));
+            if (us < best) {
+                best = us, p.rest = rest;
+                p.cut_m = cols ? 0 : (int)cut, p.cut_n = cols ? (int)cut : 0;
+                cut_cfg = c;
+            }
         }
-    p.splits = (K + p.kchunk - 1) / p.kchunk;
-    if (p.splits > 1) p.part_bytes = (size_t)p.splits * M * N * sizeof(float);
+    if (cut_cfg >= 0) p.main = {cut_cfg, 1, steps * SPLIT_STEP};
+    const size_t rm = M - p.cut_m, rn = N - p.cut_n;  // of the rest
+    const bool cut = p.cut_m || p.cut_n;
+    const int splits = cut ? p.rest.splits : p.main.splits;  // a cut plan's main launch is not split
+    if (splits > 1) p.part_bytes = (size_t)splits * rm * rn * sizeof(float);
     p.op_bytes = SplitLayout(M, N, K).bytes;
     return p;
 }
@@ -577,21 +622,38 @@ hipError_t launch_sgemm_f16(const SgemmF16Plan &p, bool a_kcontig, bool b_kconti
     };
     hipError_t e = split_operands(job(A, lda, M, a_kcontig, L.a, ea, L.pa), job(B, ldb, N, b_kcontig, L.b, eb, L.pb), K, s);
     if (e != hipSuccess) return e;
-    const bool split = p.splits > 1;
-    SplitGemmArgs a{o + L.a, o + L.b, ea, eb, A, B, a_kcontig ? lda : 1, a_kcontig ? 1 : lda, b_kcontig ? ldb : 1,
-                    b_kcontig ? 1 : ldb, split ? nullptr : bias, split ? static_cast<float *>(ws.buf) : C,
-                    split ? N : ldc, M, N, K, split ? 0 : accumulate, p.kchunk, aux_in, aux_out, ld_aux};
-    const int ge = split ? EPI_NONE : epi;
-    if (p.cfg == SPLIT_256x256) gemm_launch<256, 256, 2, 1, 2, 4, 4, 1>(ge, p.splits, a, s);
-    else if (p.cfg == SPLIT_256x128) gemm_launch<256, 128, 3, 1, 4, 2, 1, 1>(ge, p.splits, a, s);
-    else if (p.cfg == SPLIT_128x128) gemm_launch<128, 128, 2, 1, 2, 2, 1, 2>(ge, p.splits, a, s);
-    else if (p.cfg == SPLIT_128x128_KG2) gemm_launch<128, 128, 2, 2, 2, 2, 1, 1>(ge, p.splits, a, s);
-    else if (p.cfg == SPLIT_256x192) gemm_launch<256, 192, 2, 1, 4, 2, 2, 1>(ge, p.splits, a, s);
-    else gemm_launch<64, 128, 3, 2, 1, 4, 1, 1>(ge, p.splits, a, s);
-    e = hipGetLastError();
-    if (e != hipSuccess || !split) return e;
-    return launch_splitk_reduce(static_cast<const float *>(ws.buf), p.splits, M, N, bias, C, ldc, accumulate, epi,
-                                aux_in, aux_out, ld_aux, s);
+    const long sam = a_kcontig ? lda : 1, sak = a_kcontig ? 1 : lda, sbn = b_kcontig ? ldb : 1, sbk = b_kcontig ? 1 : ldb;
+    // rows [m0, m0 + rows) and columns [n0, n0 + cols), m0 and n0 multiples of 8
+    auto part = [&](const SgemmF16Part &q, int m0, int rows, int n0, int cols) {
+        const bool split = q.splits > 1;
+        const long unit = (long)split_units(K) * (SPLIT_UNIT / 8), at = (long)m0 * ld_aux + n0;
+        float *c = C + (long)m0 * ldc + n0;
+        const float *bi = bias ? bias + n0 : nullptr, *in = aux_in ? aux_in + at : nullptr;
+        float *out = aux_out ? aux_out + at : nullptr;
+        SplitGemmArgs a{o + L.a + m0 * unit, o + L.b + n0 * unit, ea + m0, eb + n0, A + m0 * sam, B + n0 * sbn, sam, sak,
+                        sbn, sbk, split ? nullptr : bi, split ? static_cast<float *>(ws.buf) : c, split ? cols : ldc,
+                        rows, cols, K, split ? 0 : accumulate, q.kchunk, in, out, ld_aux};
+        const int ge = split ? EPI_NONE : epi;
+        if (q.cfg == SPLIT_256x256) gemm_launch<256, 256, 2, 1, 2, 4, 4, 1>(ge, q.splits, a, s);
+        else if (q.cfg == SPLIT_256x128) gemm_launch<256, 128, 3, 1, 4, 2, 1, 1>(ge, q.splits, a, s);
+        else if (q.cfg == SPLIT_128x128) gemm_launch<128, 128, 2, 1, 2, 2, 1, 2>(ge, q.splits, a, s);
+        else if (q.cfg == SPLIT_128x128_KG2) gemm_launch<128, 128, 2, 2, 2, 2, 1, 1>(ge, q.splits, a, s);
+        else if (q.cfg == SPLIT_256x192) gemm_launch<256, 192, 2, 1, 4, 2, 2, 1>(ge, q.splits, a, s);
+        else gemm_launch<64, 128, 3, 2, 1, 4, 1, 1>(ge, q.splits, a, s);
+        const hipError_t g = hipGetLastError();
+        if (g != hipSuccess || !split) return g;
+        return launch_splitk_reduce(static_cast<const float *>(ws.buf), q.splits, rows, cols, bi, c, ldc, accumulate, epi,
+                                    in, out, ld_aux, s);
+    };
+    if (p.cut_m) {
+        e = part(p.main, 0, p.cut_m, 0, N);
+        return e != hipSuccess ? e : part(p.rest, p.cut_m, M - p.cut_m, 0, N);
+    }
+    if (p.cut_n) {
+        e = part(p.main, 0, M, 0, p.cut_n);
+        return e != hipSuccess ? e : part(p.rest, 0, M, p.cut_n, N - p.cut_n);
+    }
+    return part(p.main, 0, M, 0, N);
 }
 
 }  // namespace pcl
