@@ -12,6 +12,7 @@
 // adds their mean, summed in a fixed order, into *loss. Columns [V, pad) of dl
 // are written as zeros so a padded dl can feed K-padded products.
 #include "internal.h"
+#include "split_units.h"
 
 namespace pcl {
 namespace {
@@ -138,10 +139,10 @@ __global__ __launch_bounds__(CE_NT) void ce_rows_kernel(const float *logits, lon
 }
 
 // f over the block's values, the same on every thread.
-template <typename F>
-__device__ __forceinline__ float ce_block(float v, float *red, F f) {
+template <typename T, typename F>
+__device__ __forceinline__ T ce_block(T v, T *red, F f) {
 #pragma unroll
-    for (int sh = 32; sh > 0; sh >>= 1) v = f(v, __shfl_xor(v, sh));
+    for (int sh = 32; sh > 0; sh >>= 1) v = f(v, (T)__shfl_xor(v, sh));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     v = red[0];
@@ -156,27 +157,47 @@ __device__ __forceinline__ float ce_block(float v, float *red, F f) {
 // stores. The row has a scalar head up to its first 16-byte boundary
 // and a scalar tail, together at most 6 elements, one more per thread. POW2: rows
 // is a power of two, and dividing by it is multiplying by its reciprocal, exactly.
-// 4096 rows of 50257: 319 us, 5.2 TB/s, about the rate of a copy; the two-pass
+// 4096 rows of 50257: 319 us, 5.2 TB/s (a copy reaches 6.2); the two-pass
 // kernel, with its second read and two exponentials per element, took 165 us more.
-template <int NV, bool POW2>
+//
+// SPLIT: the gradient's rows are also written in the two-f16 form that d_lnf's
+// product takes (bit for bit what its split pass would make of dl), while they
+// are in registers, instead of that pass's read and write. A thread's pieces
+// then lie in pairs, eight consecutive entries, and the up to seven entries past
+// the last eight are the scalar ones. The same rows: 531 us, 4.7 TB/s, against
+// 319 and 339 for the two; head with cross-entropy 4161 -> 4035 us.
+template <int NV, bool POW2, bool SPLIT>
 __global__ __launch_bounds__(CE_NT, 4) void ce_row_regs_kernel(const float *logits, long ld,
                                                                const int *__restrict__ targets, float *dl,
                                                                long ldd, int V, int pad, float rows,
-                                                               double *__restrict__ row_loss) {
+                                                               double *__restrict__ row_loss, int M, int8_t *units,
+                                                               int *ex) {
     typedef float v4f_t __attribute__((ext_vector_type(4)));
     __shared__ float red[2][CE_NT / 64];
+    __shared__ unsigned redu[CE_NT / 64];
+    __shared__ float ends[8];  // SPLIT: the entries past the last whole eight
     const int tid = threadIdx.x, row = blockIdx.x;
     const float *x = logits + (long)row * ld;
     float *o = dl + (long)row * ldd;
-    const int head = min(V, (int)((16 - (reinterpret_cast<uintptr_t>(x) & 15)) & 15) / 4);
-    const int nv = (V - head) / 4, tail = V - head - 4 * nv;
+    // this thread's piece i: lane0 + the first entry of piece i
+    auto first = [](int i) { return SPLIT ? (i >> 1) * 2 * CE_NT + (i & 1) : i * CE_NT; };
+    const int lane0 = SPLIT ? 2 * tid : tid;
+    const int nk = split_units(V);
+    if (SPLIT && row >= M) {  // rows up to the last unit's are zeros
+        const float zero[8] = {};
+        for (int k = 8 * tid; k < pad; k += 8 * CE_NT) split_store(units, nk, row, k, zero, 0, true);
+        return;
+    }
+    const int head = SPLIT ? 0 : min(V, (int)((16 - (reinterpret_cast<uintptr_t>(x) & 15)) & 15) / 4);
+    const int nv = SPLIT ? V / 8 * 2 : (V - head) / 4, tail = V - head - 4 * nv;
+    auto has = [&](int i) { return first(SPLIT ? i & ~1 : i) + lane0 < nv; };  // a pair lies in the row whole
     const int ve = tid < head ? tid : tid < head + tail ? 4 * nv + tid : -1;  // this thread's scalar element
     const v4f_t *x4 = reinterpret_cast<const v4f_t *>(x + head);
     v4f_t a[NV];
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         a[i] = v4f_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-        if (i * CE_NT + tid < nv) a[i] = (x4 + i * CE_NT)[tid];
+        if (has(i)) a[i] = (x4 + first(i))[lane0];
     }
     float ae = ve >= 0 ? x[ve] : -INFINITY;
     const int t = targets[row];
@@ -208,15 +229,56 @@ __global__ __launch_bounds__(CE_NT, 4) void ce_row_regs_kernel(const float *logi
         return POW2 ? d * r : d / rows;
     };
     if (ve >= 0) o[ve] = one(ve == t, ae);
-    const int t0 = t - head - 4 * tid;  // the target, from this thread's first piece
+    const int t0 = t - head - 4 * lane0;  // the target, from this thread's first piece
+    unsigned mag = 0;
+    if (SPLIT && tid < 8) {
+        const float d = ve >= 0 ? one(ve == t, ae) : 0.f;
+        ends[tid] = d, mag = split_mag(d);
+    }
     v4f_t *o4 = reinterpret_cast<v4f_t *>(o + head);
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         __builtin_amdgcn_sched_barrier(0);
-        const int v = 4 * CE_NT * i;
-        if (i * CE_NT + tid < nv)
-            (o4 + i * CE_NT)[tid] = v4f_t{one(v == t0, a[i][0]), one(v + 1 == t0, a[i][1]), one(v + 2 == t0, a[i][2]),
-                                          one(v + 3 == t0, a[i][3])};
+        const int v = 4 * first(i);
+        if (has(i)) {
+            a[i] = v4f_t{one(v == t0, a[i][0]), one(v + 1 == t0, a[i][1]), one(v + 2 == t0, a[i][2]),
+                         one(v + 3 == t0, a[i][3])};
+            (o4 + first(i))[lane0] = a[i];
+#pragma unroll
+            for (int e = 0; SPLIT && e < 4; e++) mag = max(mag, split_mag(a[i][e]));
+        }
+    }
+    if constexpr (SPLIT) {
+        mag = ce_block(mag, redu, [](unsigned u, unsigned v) { return max(u, v); });
+        int shift;
+        const bool finite = split_shift(mag, shift);
+        if (tid < (pad - 4 * nv) / 8) {
+            float d[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) d[e] = tid == 0 ? ends[e] : 0.f;
+            split_store(units, nk, row, 4 * nv + 8 * tid, d, shift, finite);
+        }
+        if (tid == 0) ex[row] = finite ? -shift : SPLIT_NONFINITE;
+        // the addresses of split_store, with the lane's part in 32 bits
+        int8_t *base = units + (long)(row >> 3) * nk * SPLIT_UNIT + (row & 7) * 128;
+        const unsigned lane = (8 * tid / SPLIT_BK) * SPLIT_UNIT, c = (tid & 3) * 2, key = row >> 1 & 7;
+        const unsigned at_hi = lane + ((c ^ key) << 4), at_lo = lane + (((c + 1) ^ key) << 4);
+#pragma unroll
+        for (int i = 0; i < NV; i += 2) {
+            __builtin_amdgcn_sched_barrier(0);
+            v8h hi, lo;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                _Float16 h, l;
+                split_value(a[i + e / 4][e % 4], shift, finite, h, l);
+                hi[e] = h, lo[e] = l;
+            }
+            if (has(i)) {
+                int8_t *u = base + (long)(i >> 1) * (8 * CE_NT / SPLIT_BK) * SPLIT_UNIT;
+                *reinterpret_cast<v8h *>(u + at_hi) = hi;
+                *reinterpret_cast<v8h *>(u + at_lo) = lo;
+            }
+        }
     }
     if (!(pt < 0.f)) row_loss[row] = -log((double)pt + 1e-30);
     for (int v = V + tid; v < pad; v += CE_NT) o[v] = 0.f;
@@ -246,17 +308,37 @@ hipError_t launch_cross_entropy(const float *logits, long ld, const int *targets
                       (ld - ldd) % 4 == 0;
     // 25 pieces fill the 128 registers that two workgroups per CU leave a thread
     const int pieces = (V + 4 * CE_NT - 1) / (4 * CE_NT);  // 16-byte pieces per thread
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)M), dim3(CE_NT), 0, s, logits, ld, targets, dl, ldd, V, pad,
+    if (!same || pieces > 25) {
+        hipLaunchKernelGGL(ce_rows_kernel, dim3((unsigned)M), dim3(CE_NT), 0, s, logits, ld, targets, dl, ldd, V, pad,
                            (float)rows, row_loss);
+        return hipGetLastError();
+    }
+    auto launch = [&](auto general, auto pow2) {
+        hipLaunchKernelGGL(rows & (rows - 1) ? general : pow2, dim3((unsigned)M), dim3(CE_NT), 0, s, logits, ld, targets,
+                           dl, ldd, V, pad, (float)rows, row_loss, M, nullptr, nullptr);
     };
-    auto regs = [&](auto general, auto pow2) { rows & (rows - 1) ? launch(general) : launch(pow2); };
-    if (!same || pieces > 25) launch(ce_rows_kernel);
-    else if (pieces <= 1) regs(ce_row_regs_kernel<1, false>, ce_row_regs_kernel<1, true>);
-    else if (pieces <= 4) regs(ce_row_regs_kernel<4, false>, ce_row_regs_kernel<4, true>);
-    else if (pieces <= 8) regs(ce_row_regs_kernel<8, false>, ce_row_regs_kernel<8, true>);
-    else if (pieces <= 16) regs(ce_row_regs_kernel<16, false>, ce_row_regs_kernel<16, true>);
-    else regs(ce_row_regs_kernel<25, false>, ce_row_regs_kernel<25, true>);
+    if (pieces <= 1) launch(ce_row_regs_kernel<1, false, false>, ce_row_regs_kernel<1, true, false>);
+    else if (pieces <= 4) launch(ce_row_regs_kernel<4, false, false>, ce_row_regs_kernel<4, true, false>);
+    else if (pieces <= 8) launch(ce_row_regs_kernel<8, false, false>, ce_row_regs_kernel<8, true, false>);
+    else if (pieces <= 16) launch(ce_row_regs_kernel<16, false, false>, ce_row_regs_kernel<16, true, false>);
+    else launch(ce_row_regs_kernel<25, false, false>, ce_row_regs_kernel<25, true, false>);
+    return hipGetLastError();
+}
+
+hipError_t launch_cross_entropy_split(const CeRows &c, int M, int V, int8_t *units, int *ex, hipStream_t s) {
+    if (M <= 0) return hipSuccess;
+    static_assert(CE_SPLIT_PAD == 26 * 4 * CE_NT, "pieces of the largest kernel");
+    if (c.pad > CE_SPLIT_PAD || c.pad != split_units(V) * SPLIT_BK || (reinterpret_cast<uintptr_t>(c.logits) & 15))
+        return hipErrorInvalidValue;
+    const int pieces = (c.pad + 4 * CE_NT - 1) / (4 * CE_NT);
+    auto launch = [&](auto general, auto pow2) {
+        hipLaunchKernelGGL(c.rows & (c.rows - 1) ? general : pow2, dim3((unsigned)(M + 7) / 8 * 8), dim3(CE_NT), 0, s,
+                           c.logits, (long)c.pad, c.targets, c.logits, (long)c.pad, V, c.pad, (float)c.rows, c.row_loss,
+                           M, units, ex);
+    };
+    if (pieces <= 8) launch(ce_row_regs_kernel<8, false, true>, ce_row_regs_kernel<8, true, true>);
+    else if (pieces <= 16) launch(ce_row_regs_kernel<16, false, true>, ce_row_regs_kernel<16, true, true>);
+    else launch(ce_row_regs_kernel<26, false, true>, ce_row_regs_kernel<26, true, true>);
     return hipGetLastError();
 }
 

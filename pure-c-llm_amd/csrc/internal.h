@@ -27,6 +27,16 @@ struct GemvPlan {
 };
 
 // ---- FP32 GEMM (sgemm.hip) ----
+// Rows of logits (rows of pad floats, 16-byte aligned, pad = V rounded up to 64 and
+// at most CE_SPLIT_PAD) that a product takes as its K-contiguous op(A) after the
+// cross-entropy of launch_cross_entropy, in place, which then splits them too.
+constexpr int CE_SPLIT_PAD = 53248;
+struct CeRows {
+    float *logits = nullptr;
+    const int *targets = nullptr;
+    int pad = 0, rows = 0;
+    double *row_loss = nullptr;
+};
 // The same product on the f16 matrix cores (sgemm_split.hip): tile and K split,
 // bytes of the split operands (0: the shape has no such form) and of the
 // partial products. With cut_m or cut_n, rows or columns from there on are a
@@ -38,6 +48,7 @@ struct SgemmF16Plan {
     SgemmF16Part main, rest;
     int cut_m = 0, cut_n = 0;
     size_t op_bytes = 0, part_bytes = 0;
+    CeRows ce;  // with logits: op(A) is the cross-entropy's gradient of them
 };
 // Tile configuration and K split chosen for a shape; with splits > 1 the
 // partial products ([splits][M][N] fp32, part_bytes) go to the workspace and a
@@ -139,6 +150,9 @@ hipError_t launch_decode_argmax(const float *logits, int V, int *tokpos, int *ou
 hipError_t launch_cross_entropy(const float *logits, long ld, const int *targets, float *dl,
                                 long ldd, int M, int V, int pad, int rows, double *row_loss,
                                 hipStream_t s);
+// The same for M rows of c over a vocabulary of V, and the gradient's units and
+// exponents (split_units.h; rows up to a multiple of 8).
+hipError_t launch_cross_entropy_split(const CeRows &c, int M, int V, int8_t *units, int *ex, hipStream_t s);
 // *loss += (float)(sum of row_loss[0..M) / rows)
 hipError_t launch_ce_loss(const double *row_loss, int M, int rows, float *loss, hipStream_t s);
 

@@ -1640,12 +1640,20 @@ int pcl_head_ce(const float *lnf, const float *wte, const int *targets, int M, i
         const float *x = lnf + (size_t)m0 * D;
         // train.c:412-423 on the chunk, then :449-465 in place
         PCL_OK_OR_RETURN(pcl_sgemm(PCL_OP_N, PCL_OP_T, mm, V, D, x, D, wte, D, nullptr, 0, lg, L, s));
-        HIP_OK(pcl::launch_cross_entropy(lg, ldp, targets + m0, lg, ldp, mm, V, L, M, rl + m0, s));
         // the vocabulary in two parts on the f32 matrix cores, whole on the f16 ones
-        const bool f16 = f16_pays(pcl::plan_sgemm(mm, D, V), PCL_OP_N, PCL_OP_N, mm, D, V, lg, L, wte, D);
+        pcl::SgemmPlan px = pcl::plan_sgemm(mm, D, V);
+        const bool f16 = f16_pays(px, PCL_OP_N, PCL_OP_N, mm, D, V, lg, L, wte, D);
         const int Vm = f16 ? V : V / 64 * 64, Vr = V - Vm;
-        if (d_lnf) {  // train.c:426-435 (set): K = V
-            float *dx = d_lnf + (size_t)m0 * D;
+        float *dx = d_lnf ? d_lnf + (size_t)m0 * D : nullptr;
+        int st = 1;
+        if (dx && f16 && L <= pcl::CE_SPLIT_PAD) {  // the cross-entropy as d_lnf's split pass
+            px.f16.ce = {lg, targets + m0, L, M, rl + m0};
+            st = sgemm_f16(px, PCL_OP_N, PCL_OP_N, mm, D, V, lg, L, wte, D, nullptr, 0, dx, D, s);
+            if (st != PCL_OK && st != 1) return st;
+        }
+        if (st != PCL_OK)
+            HIP_OK(pcl::launch_cross_entropy(lg, ldp, targets + m0, lg, ldp, mm, V, L, M, rl + m0, s));
+        if (dx && st != PCL_OK) {  // train.c:426-435 (set): K = V
             PCL_OK_OR_RETURN(pcl_sgemm(PCL_OP_N, PCL_OP_N, mm, D, Vm, lg, L, wte, D, nullptr, 0, dx, D, s));
             if (Vr)
                 PCL_OK_OR_RETURN(pcl_sgemm(PCL_OP_N, PCL_OP_N, mm, D, Vr, lg + Vm, L, wte + (size_t)Vm * D,

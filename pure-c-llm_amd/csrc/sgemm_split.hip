@@ -29,44 +29,9 @@
 // of consecutive memory. The GEMM kernel streams the units through an LDS ring.
 #include "internal.h"
 #include "sgemm_common.h"
+#include "split_units.h"
 
 namespace pcl {
-
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-
-constexpr int SPLIT_BK = 32;                // k per unit
-constexpr int SPLIT_KUNITS = 2;             // operands are padded to this many units of k
-constexpr int SPLIT_UNIT = 1024;            // bytes of 8 rows x 32 k
-constexpr int SPLIT_NONFINITE = 1 << 28;    // exponent of a row with inf or NaN
-
-__host__ __device__ constexpr int split_units(int K) {
-    return (K + SPLIT_BK * SPLIT_KUNITS - 1) / (SPLIT_BK * SPLIT_KUNITS) * SPLIT_KUNITS;
-}
-
-// A row's scale from the bits of its largest |a|: shift to add to the exponents
-// of its elements, or none if it is not finite.
-__device__ __forceinline__ bool split_shift(unsigned amax, int &shift) {
-    if (amax >= 0x7f800000u) return shift = 0, false;
-    if (amax == 0) return shift = 0, true;
-    const int e = amax >= 0x00800000u ? (int)(amax >> 23) - 127 : -118 - __clz((int)amax);
-    return shift = 14 - e, true;
-}
-
-// Eight consecutive k of one row: hi and lo at the unit's two chunks.
-__device__ __forceinline__ void split_store(int8_t *P, int nk, int row, int k, const float (&a)[8], int shift,
-                                            bool finite) {
-    v8h hi, lo;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const float x = finite ? ldexpf(a[e], shift) : 0.f;
-        hi[e] = (_Float16)x;
-        lo[e] = (_Float16)(x - (float)hi[e]);
-    }
-    int8_t *u = P + ((long)(row >> 3) * nk + (k >> 5)) * SPLIT_UNIT + (row & 7) * 128;
-    const int c = (k >> 3 & 3) * 2, key = row >> 1 & 7;
-    *reinterpret_cast<v8h *>(u + ((c ^ key) << 4)) = hi;
-    *reinterpret_cast<v8h *>(u + (((c + 1) ^ key) << 4)) = lo;
-}
 
 // One operand to split: element (row, k) at X[row * ld + k] (kcontig) or X[k * ld + row].
 struct SplitJob {
@@ -87,7 +52,6 @@ __device__ __forceinline__ v4f split_load4(const float *x, int i, int n, bool ve
     for (int e = 0; e < 4; e++) v[e] = i + e < n ? x[i + e] : 0.f;
     return v;
 }
-__device__ __forceinline__ unsigned split_mag(float x) { return __float_as_uint(x) & 0x7fffffffu; }
 
 // Operand with consecutive k: NT threads per row, each G groups of 8 k in
 // registers, so the operand is read once (rows of up to 8 NT G floats; MULTI:
@@ -620,7 +584,11 @@ hipError_t launch_sgemm_f16(const SgemmF16Plan &p, bool a_kcontig, bool b_kconti
         return SplitJob{X, ld, rows, kc, (reinterpret_cast<uintptr_t>(X) & 15) == 0 && ld % 4 == 0, o + P, ex,
                         reinterpret_cast<unsigned *>(o + part), 0};
     };
-    hipError_t e = split_operands(job(A, lda, M, a_kcontig, L.a, ea, L.pa), job(B, ldb, N, b_kcontig, L.b, eb, L.pb), K, s);
+    hipError_t e = hipSuccess;
+    const bool ce = p.ce.logits != nullptr;  // splits op(A) itself
+    if (ce) e = launch_cross_entropy_split(p.ce, M, K, o + L.a, ea, s);
+    if (e != hipSuccess) return e;
+    e = split_operands(job(A, lda, ce ? 0 : M, a_kcontig, L.a, ea, L.pa), job(B, ldb, N, b_kcontig, L.b, eb, L.pb), K, s);
     if (e != hipSuccess) return e;
     const long sam = a_kcontig ? lda : 1, sak = a_kcontig ? 1 : lda, sbn = b_kcontig ? ldb : 1, sbk = b_kcontig ? 1 : ldb;
     // rows [m0, m0 + rows) and columns [n0, n0 + cols), m0 and n0 multiples of 8
